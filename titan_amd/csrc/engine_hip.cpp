@@ -473,14 +473,15 @@ eh_status run_tiles(eh_context* c, eh_stream stream, const tiles_args& a, const 
 }
 
 // Splits: aim for enough workgroups to fill 256 CUs several times over, with
-// at most kMaxSplits splits and none beyond the largest.
+// at most kMaxSplits splits, in whole rounds; the largest split (the limit every
+// call checks) is whole chunks only.
 uint64_t auto_tps(uint64_t batch, const decode_kernel& dk, uint64_t max_ctx, uint64_t block_tokens,
                   uint64_t target_wgs = 1024) {
-    const uint64_t chunk = dk.round;
+    const uint64_t round = dk.round;
     uint64_t tps = div_ceil(batch * dk.units * (max_ctx ? max_ctx : 1), target_wgs);
-    tps = std::max<uint64_t>((tps + chunk / 2) / chunk, 1) * chunk;  // nearest chunk multiple
-    while (div_ceil(max_ctx ? max_ctx : 1, tps) > kMaxSplits) tps += chunk;
-    return std::min(tps, max_tps(block_tokens, chunk, dk.rows));
+    tps = std::max<uint64_t>((tps + round / 2) / round, 1) * round;  // nearest multiple
+    while (div_ceil(max_ctx ? max_ctx : 1, tps) > kMaxSplits) tps += round;
+    return std::min(tps, max_tps(block_tokens, dk.chunk, dk.rows));
 }
 
 // Checks shared by the single-sequence attention entry points
@@ -1278,8 +1279,7 @@ eh_status eh_decode_plan(uint32_t kv_dtype, uint32_t batch, uint32_t n_head, uin
     // 2048, 42.3 at 4096), but none under 128 tokens, whose merge costs more than
     // it spreads (f32, 14/2 heads of 64: 15.1 us at 128, 17.6 at 64).
     uint64_t tps = hint      ? div_ceil(hint, dk.chunk) * dk.chunk
-                   : dk.rows ? std::max<uint64_t>(auto_tps(batch, dk, max_ctx, block_tokens, 2048),
-                                                  std::min<uint64_t>(128, max_tps(block_tokens, dk.round, true)))
+                   : dk.rows ? std::max<uint64_t>(auto_tps(batch, dk, max_ctx, block_tokens, 2048), 128)
                              : auto_tps(batch, dk, max_ctx, block_tokens);
     while (div_ceil(max_ctx ? max_ctx : 1, tps) > kMaxSplits) tps *= 2;
     if (tps > max_tps(block_tokens, dk.chunk, dk.rows))
