@@ -158,6 +158,15 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// Orders a wave's LDS accesses around it, for the compiler: lanes read what other
+// lanes of the wave wrote.  The hardware keeps a wave's LDS accesses in order; no
+// instruction is emitted.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 __device__ __forceinline__ uint32_t uni(uint32_t v) {
     return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
 }
@@ -490,6 +499,7 @@ __device__ __forceinline__ void decode_tiles(
             const uint32_t i = lane + 64 * u;
             if (i < (uint32_t)NQ4) reinterpret_cast<float4*>(qst)[i] = v[u];
         }
+        wave_lds_order();
     }
     // q of sequence b: staged (LDS) or, past the staged ones, fetched now.
     // Contraction index of MFMA step st, lane (g, x): dims 32 st + 8 g + e for
@@ -679,7 +689,9 @@ __device__ __forceinline__ void decode_tiles(
             }
         }
 
-        // K tile rows into LDS as they are (they come back in the operand layout)
+        // K tile rows into LDS as they are (they come back in the operand layout),
+        // behind every lane's reads of the last tile
+        wave_lds_order();
         static_for<0, NREG>([&](auto Rc) {
             constexpr int j = decltype(Rc)::value;
             *reinterpret_cast<u32x4*>(kt + (F8 ? (lane >> 3) + 8 * j : 4 * g + j) * KROW +
@@ -721,6 +733,7 @@ __device__ __forceinline__ void decode_tiles(
             });
         }
 
+        wave_lds_order();
         // S = K Q^T: lane (g, x) receives tokens 4g..4g+3 of head x; A operand:
         // token x, 16-bit dims 32 st + 8 g .., E4M3 codes 32 g + 8 st ..
         f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
