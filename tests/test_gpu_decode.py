@@ -826,3 +826,83 @@ def test_row_kernels_heads_of_any_magnitude(dev, dtype, hd):
     # 1e3 * 2^-24 * 8 in the exponent; the others are small or one-hot
     assert (err < 5e-4).all(), err
     assert (err[[0, 2, 4, 6, 8]] < 1e-5).all(), err
+
+
+LONG_TABLES = [  # (n_head, n_kv, head_dim, block_tokens, table entries)
+    (32, 32, 128, 16, 8192), (14, 2, 64, 8, 8192), (12, 3, 128, 4, 20000), (16, 1, 64, 32, 3000)]
+
+
+@pytest.mark.parametrize("dtype", [KvDataType.F32, KvDataType.F16, KvDataType.BF16])
+@pytest.mark.parametrize("shape", LONG_TABLES, ids=lambda s: "x".join(map(str, s)))
+def test_device_position_far_below_the_table(dev, dtype, shape):
+    """Device positions from one token up to thousands under tables of up to
+    131072 tokens: the splits are cut by the live length (around a round, a whole
+    number of them, the last slot), table entries behind it name no page, the
+    fused step writes its row."""
+    n_head, n_kv, hd, bt, entries = shape
+    rng = np.random.default_rng(sum(shape))
+    td = {KvDataType.F32: torch.float32, KvDataType.F16: torch.float16,
+          KvDataType.BF16: torch.bfloat16}[dtype]
+    most = 4200
+    nb = -(-most // bt)
+    table = np.full(entries, 0xFFFFFFFF, np.uint32)
+    table[:nb] = rng.permutation(nb)
+    rows = torch.from_numpy(rng.standard_normal((most, 2, n_kv * hd)).astype(np.float32)).to(td)
+    pool = torch.zeros((nb * bt, 2, n_kv * hd), dtype=td)
+    p = np.arange(most)
+    where = torch.from_numpy(table[p // bt].astype(np.int64) * bt + p % bt)
+    pool[where] = rows
+    r = rows.float().numpy().reshape(most, 2, n_kv, hd)
+    pa = PagedAttention(0)
+    dt = i32(table, dev)
+    q = rng.standard_normal((n_head, hd)).astype(np.float32)
+    dq = torch.from_numpy(q).to(dev)
+    for pos in (0, 63, 64, 127, 128, 1000, 2047, 2048, 4159):
+        want = _sdpa64(q, r[:pos + 1, 0], r[:pos + 1, 1])
+        dp = pool.reshape(-1).to(dev)
+        out = torch.full((n_head, hd), float("nan"), device=dev)
+        pa.launch_flash_decoding(None, dq, dp, dt, out, n_head, n_kv, hd, bt, pos + 1, pos, True,
+                                 i32([pos], dev), kv_dtype=dtype)
+        parity.check_close(out.cpu().numpy(), want, f32=True, what=f"position {pos}")
+        hole = pool.clone()
+        hole[where[pos]] = float("nan")
+        dp = hole.reshape(-1).to(dev)
+        out.fill_(float("nan"))
+        pa.append_flash_decoding(None, rows[pos, 0].to(dev), rows[pos, 1].to(dev), dq, dp, dt, out, n_head,
+                                 n_kv, hd, bt, pos, i32([pos], dev), dtype)
+        parity.check_close(out.cpu().numpy(), want, f32=True, what=f"fused, position {pos}")
+        assert torch.equal(dp.cpu(), pool.reshape(-1)), pos
+
+
+def test_device_position_costs_by_its_length(dev):
+    """A step at 4000 live tokens under a table of 131072 takes about what it takes
+    under a table of its own (f32, 32/8 heads of 128: 12 us in both; splits cut by
+    the capacity alone took 116): at most three times."""
+    n_head, n_kv, hd, bt, live = 32, 8, 128, 16, 4000
+    nb = live // bt
+    pool = torch.randn(nb * bt * 2 * n_kv * hd, device=dev)
+    q = torch.randn((n_head, hd), device=dev)
+    out = torch.empty_like(q)
+    pos = i32([live - 1], dev)
+    pa = PagedAttention(0)
+    took = []
+    for entries in (nb, 8192):
+        table = np.full(entries, 0xFFFFFFFF, np.uint32)
+        table[:nb] = np.random.default_rng(3).permutation(nb)
+        dt = i32(table, dev)
+        pa.launch_flash_decoding(None, q, pool, dt, out, n_head, n_kv, hd, bt, live, live - 1, True, pos)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            for _ in range(20):
+                pa.launch_flash_decoding(None, q, pool, dt, out, n_head, n_kv, hd, bt, live, live - 1, True, pos)
+        best = float("inf")
+        for _ in range(5):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            g.replay()
+            b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b))
+        took.append(best)
+    assert took[1] < 3 * took[0], took

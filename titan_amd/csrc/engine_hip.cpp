@@ -249,7 +249,8 @@ struct decode_kernel {
     uint32_t g = 1;       // head-major: compiled head-group width
     uint32_t chunks = 1;  // workgroups per (split, kv head, sequence)
     uint64_t chunk = 1;   // a split is a multiple of this many tokens
-    uint64_t round = 1;   // tokens one pass of the workgroup's waves takes (planned splits)
+    uint64_t round = 1;   // tokens one pass of the workgroup's waves takes (planned splits, and
+                          // the row kernels' own ones: live_tps in decode_len.h)
     uint64_t units = 1;   // workgroups per (split, sequence)
 };
 
@@ -320,17 +321,26 @@ eh_status run_decode(eh_context* c, eh_stream stream, const decode_args& a) {
     const hipModule_t mod = c->mod_decode[dt_index(a.kv_dtype)];
     const dim3 grid = dk.rows ? dim3(a.batch, a.n_head_kv * dk.chunks, a.max_splits)
                               : dim3(a.max_splits, a.n_head_kv * dk.chunks, a.batch);
-    eh_status st = launch(c, dk.rows ? c->mod_rows : mod, name, grid, dim3(kDecodeThreads), stream,
-                          a.q, (const uint8_t*)a.pool, a.bt, a.bt_stride, a.lens_ptr, a.lens_mode,
-                          a.seq_tokens, a.query_pos, a.causal, a.out, a.part_acc, a.part_ml, a.n_head,
-                          a.n_head_kv, a.block_tokens, bt_shift, a.tps, a.max_splits, scale_log2,
-                          a.n_blocks, (const uint8_t*)a.new_k, (const uint8_t*)a.new_v);
+    // device position: contexts from which the row kernels cut shorter splits (live_tps)
+    const uint32_t shorter =
+        dk.rows && a.lens_mode == 1 && a.tps > dk.round
+            ? (uint32_t)std::min<uint64_t>((uint64_t)a.max_splits * (a.tps - dk.round) + 1, 0xFFFFFFFFu)
+            : 0u;
+    auto split = [&](hipModule_t m, auto... more) {
+        return launch(c, m, name, grid, dim3(kDecodeThreads), stream, a.q, (const uint8_t*)a.pool, a.bt,
+                      a.bt_stride, a.lens_ptr, a.lens_mode, a.seq_tokens, a.query_pos, a.causal, a.out,
+                      a.part_acc, a.part_ml, a.n_head, a.n_head_kv, a.block_tokens, bt_shift, a.tps,
+                      a.max_splits, scale_log2, a.n_blocks, (const uint8_t*)a.new_k,
+                      (const uint8_t*)a.new_v, more...);
+    };
+    eh_status st = dk.rows ? split(c->mod_rows, shorter) : split(mod);
     if (st != EH_OK || a.max_splits <= 1) return st;
     return launch(c, mod, "eh_decode_merge",
                   dim3((uint32_t)div_ceil((uint64_t)a.n_head * a.head_dim, 64), a.batch), dim3(256),
                   stream,
                   (const float*)a.part_acc, (const float*)a.part_ml, a.out, a.lens_ptr, a.lens_mode,
-                  a.seq_tokens, a.query_pos, a.causal, a.n_head, a.head_dim, a.tps, a.max_splits);
+                  a.seq_tokens, a.query_pos, a.causal, a.n_head, a.head_dim, a.tps, a.max_splits,
+                  (uint32_t)std::max(log2_exact(dk.round), 0), shorter);
 }
 
 // ---- token-balanced decode (eh_decode_tiles_*, paged_decode_tiles.hip)
@@ -1128,7 +1138,10 @@ static eh_status single_seq_attention(eh_context* c, eh_stream stream, uint32_t 
     // One sequence: a quarter of the workgroups per kv head for the row kernels,
     // whose merge then reads fewer partials (32/8 heads of 128 at 8191 tokens,
     // f16: 256 / 512 / 1024 workgroups 12.3 / 13.8 / 13.8 us; f32 8000 tokens
-    // 17.4 / 19.5 / 25.2).
+    // 17.4 / 19.5 / 25.2).  Under a device position this covers the table's capacity;
+    // the kernels cut a shorter context by its own length (32/8 heads of 128, f32, 4000
+    // tokens under a table of 131072: 116 us by the capacity, 12.2 so, 11.9 under a
+    // table of its own; f16 28.9, 8.8, 8.4).
     uint64_t tps = auto_tps(1, dk, cap, block_tokens, dk.rows ? 256 : 1024);
     if (single_pass && cap <= most)
         tps = std::max<uint64_t>(div_ceil(cap, chunk), 1) * chunk;

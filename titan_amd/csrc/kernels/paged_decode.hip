@@ -40,6 +40,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "decode_len.h"
+
 namespace {
 
 constexpr int NW = 4;  // waves per workgroup
@@ -123,28 +125,6 @@ __device__ __forceinline__ float group_sum(float v) {
     if constexpr (N >= 32) v += __shfl_xor(v, 16, 64);
     if constexpr (N >= 64) v += __shfl_xor(v, 32, 64);
     return v;
-}
-
-struct len_src {
-    const uint32_t* ptr;  // device lengths or position
-    uint32_t mode;        // 0: host scalars, 1: *ptr is the query position, 2: ptr[b] = tokens
-    uint32_t seq_tokens, query_pos, causal;
-};
-
-__device__ __forceinline__ uint32_t live_tokens(const len_src& L, uint32_t b) {
-    if (L.mode == 2) return L.ptr[b];
-    if (L.mode == 1) return L.ptr[0] + 1u;  // paged_attention.cu:21-24
-    uint32_t n = L.seq_tokens;
-    if (L.causal && L.query_pos + 1u < n) n = L.query_pos + 1u;
-    return n;
-}
-
-// Splits covering n tokens, capped by the launched grid.  Callers size the
-// grid so that n <= max_splits * tps; the cap only keeps a violating length
-// inside the workspace.
-__device__ __forceinline__ uint32_t split_count(uint32_t n, uint32_t tps, uint32_t max_splits) {
-    const uint32_t s = n / tps + (n % tps != 0u);
-    return s < max_splits ? s : max_splits;
 }
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
@@ -412,7 +392,8 @@ __device__ __forceinline__ void decode_split(
 extern "C" __global__ __launch_bounds__(256) void eh_decode_merge(
     const float* __restrict__ part_acc, const float* __restrict__ part_ml, float* __restrict__ out,
     const uint32_t* lens_ptr, uint32_t lens_mode, uint32_t seq_tokens, uint32_t query_pos,
-    uint32_t causal, uint32_t n_head, uint32_t head_dim, uint32_t tps, uint32_t max_splits) {
+    uint32_t causal, uint32_t n_head, uint32_t head_dim, uint32_t tps, uint32_t max_splits,
+    uint32_t round_log2, uint32_t shorter) {
     constexpr int NB = 8;
     __shared__ float sM[NW][64], sL[NW][64], sA[NW][64];
     const len_src L{lens_ptr, lens_mode, seq_tokens, query_pos, causal};
@@ -442,7 +423,7 @@ extern "C" __global__ __launch_bounds__(256) void eh_decode_merge(
     };
     fetch(0, max_splits);
     const uint32_t n = live_tokens(L, b);
-    const uint32_t nsplit = split_count(n, tps, max_splits);
+    const uint32_t nsplit = split_count(n, live_tps(n, tps, max_splits, round_log2, shorter), max_splits);
     if (n == 0 || nsplit <= 1) return;  // the split kernel wrote the output (uniform)
     float M = -INFINITY, Ls = 0.0f, A = 0.0f;
     for (uint32_t s0 = 0; s0 + wave < nsplit; s0 += NW * NB) {
