@@ -46,7 +46,7 @@ def test_code_objects_contain_launched_kernels():
         for k in ("eh_append_kv_c", "eh_gather_kv_c", "eh_copy_pages_c"):
             assert f"{k}{ch}".encode() in kv
     for k in ("eh_remap_block_tables", "eh_page_refcounts", "eh_fill_u32", "eh_append_kv_e4m3",
-              "eh_gather_kv_e4m3", "eh_kv_e4m3_scales", "eh_kv_e4m3_scales_rows",
+              "eh_gather_kv_e4m3", "eh_kv_e4m3_scales", "eh_kv_e4m3_scales_seed", "eh_kv_e4m3_scales_rows",
               "eh_stream_pages_d1",
               "eh_stream_pages_d2", "eh_stream_pages_heads"):
         assert k.encode() in kv

@@ -279,6 +279,72 @@ def test_e4m3_scales_many_rows(dev, n_kv, hd, n):
     assert np.array_equal(vs.cpu().numpy().view(np.uint32), e4m3_scales_np(v, n_kv, hd).view(np.uint32))
 
 
+@pytest.mark.parametrize("n_kv,hd,n", [
+    (2, 128, 161),                     # the first size of two launches
+    (12, 96, 400), (3, 1500, 30),      # heads across two column blocks, and three
+    (8, 128, 3000), (70, 128, 200),    # many workgroups a head; nine column blocks
+])
+def test_e4m3_scales_dead_heads(dev, n_kv, hd, n):
+    """Heads with no finite nonzero element in the rows that seed the two-launch
+    scan: none at all (scale 1, also where zeros and non-finite values mix), the
+    only one in the first row behind them, in the last row, and a scale of 1 by a
+    largest element of 448; first, last and block-straddling heads among them."""
+    rng = np.random.default_rng(n_kv)
+    k, v = (rng.standard_normal((n, n_kv, hd)).astype(np.float32) for _ in range(2))
+    behind = 1024 // (hd // 4)               # the first row behind the seeding round
+    for h in {0, n_kv - 1, 1024 // hd % n_kv}:
+        k[:, h] = 0.0
+        v[:, h] = np.float32(np.nan)
+        v[::3, h] = 0.0
+    if n_kv > 4:
+        k[:, 2] = 0.0
+        k[min(behind + 1, n - 1), 2, hd - 1] = -7.0
+        k[:, 3] = 0.0
+        k[-1, 3, 0] = 1e-42                 # subnormal: the FLT_MIN floor
+        v[:, 2] = 0.0
+        v[n - 2, 2, 1] = 448.0
+    layout = PagedKvLayout(4, 16, n_kv * hd, KvDataType.FP8)
+    k, v = k.reshape(n, -1), v.reshape(n, -1)
+    for _ in range(2):                      # and over the scales of a call before
+        ks, vs = (torch.full((n_kv,), 3e-40, device=dev) for _ in range(2))
+        for _ in range(2):
+            PagedKvGpu(0).e4m3_scales(None, layout, torch.from_numpy(k).to(dev), torch.from_numpy(v).to(dev),
+                                      hd, ks, vs)
+            assert np.array_equal(ks.cpu().numpy().view(np.uint32), e4m3_scales_np(k, n_kv, hd).view(np.uint32))
+            assert np.array_equal(vs.cpu().numpy().view(np.uint32), e4m3_scales_np(v, n_kv, hd).view(np.uint32))
+
+
+def test_e4m3_scales_cost_of_a_dead_head(dev):
+    """A head of zeros is read by one workgroup before the scan proper, with its loads
+    in flight: 4096 rows of 8 heads take 11 us without one and 47 with it (146 with a
+    few loads in flight); at most six times."""
+    n_kv, hd, n = 8, 128, 4096
+    layout = PagedKvLayout(4, 16, n_kv * hd, KvDataType.FP8)
+    kv = PagedKvGpu(0)
+    k, v = (torch.randn((n, n_kv * hd), device=dev) for _ in range(2))
+    ks, vs = (torch.empty(n_kv, device=dev) for _ in range(2))
+    took = []
+    for dead in (False, True):
+        if dead:
+            k.view(n, n_kv, hd)[:, 3] = 0.0
+        kv.e4m3_scales(None, layout, k, v, hd, ks, vs)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            for _ in range(20):
+                kv.e4m3_scales(None, layout, k, v, hd, ks, vs)
+        best = float("inf")
+        for _ in range(5):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            g.replay()
+            b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b))
+        took.append(best)
+    assert took[1] < 6 * took[0], took
+
+
 def test_e4m3_dynamic_scales_end_to_end(dev):
     """The FP8 spec's flow (specs/kv-compression/spec.md:8-14): scales from the
     prompt's own K/V on the device, the quantising append with them, E4M3

@@ -931,14 +931,15 @@ eh_status eh_kv_e4m3_scales(eh_context* c, eh_stream stream, const eh_kv_layout*
     // read by the whole chip.  Measured (8 heads of 128): one workgroup per
     // head 5.6 us at 4096 float4s a head and 0.75 us per 1024 more, two
     // launches 6.4 us there and 11.2 us at 131072 (241 us before).  256
-    // workgroups in all: 512 / 1024 / 2048 took 12.5 / 14.6 / 14.9 us
-    // where 256 take 11.2 (34 MB), 25 / 36 / 46 where they take 26 (134 MB) --
-    // every workgroup ends at the same few scale words.
+    // workgroups in all (rows of more than 8192 elements: 16 per column block and
+    // side): 512 / 1024 / 2048 took 12.5 / 14.6 / 14.9 us where 256 take 11.2
+    // (34 MB), 25 / 36 / 46 where they take 26 (134 MB) -- every workgroup ends at
+    // the same few scale words.
     const uint64_t quads = l->row_len / 4;
     const bool wide = n_rows * (head_dim / 4) > kScaleScanQuads && quads <= 256ull * 65535;
-    st = launch(c, c->mod_kv, "eh_kv_e4m3_scales", dim3((uint32_t)n_kv, 2), dim3(256), stream,
-                keys, values, (uint32_t)n_rows, (uint32_t)l->row_len, head_dim, k_scale, v_scale,
-                (uint32_t)wide);
+    st = launch(c, c->mod_kv, wide ? "eh_kv_e4m3_scales_seed" : "eh_kv_e4m3_scales",
+                dim3((uint32_t)n_kv, 2), dim3(wide ? 1024 : 256), stream, keys, values,
+                (uint32_t)n_rows, (uint32_t)l->row_len, head_dim, k_scale, v_scale);
     if (st || !wide) return st;
     const uint64_t side = 256 / std::min<uint64_t>(quads, 256);  // rows read side by side
     const uint64_t blocks = div_ceil(quads, 256);

@@ -244,34 +244,40 @@ __device__ __forceinline__ float e4m3_scale_of(float amax) {
 }
 }  // namespace
 
-// One workgroup per head.  Grid (n_kv, 2): y = 0 reads keys into k_scale,
-// y = 1 values into v_scale; 256 threads; head_dim % 4 == 0.  With `seed` the
-// scan ends with the first round of loads that found a finite nonzero
-// element: the scale written is then a lower bound that
-// eh_kv_e4m3_scales_rows raises, and 1 only if no row holds such an element.
-extern "C" __global__ __launch_bounds__(256) void eh_kv_e4m3_scales(
-    const float* keys, const float* values, uint32_t n_rows, uint32_t row_len, uint32_t head_dim,
-    float* k_scale, float* v_scale, uint32_t seed) {
-    constexpr int U = 4;  // loads in flight per thread
-    __shared__ float wmax[4];
-    const uint32_t h = blockIdx.x;
-    const float* src = (blockIdx.y ? values : keys) + (uint64_t)h * head_dim;
-    const uint32_t qph = head_dim / 4;  // float4s per head row
-    const uint64_t total = (uint64_t)n_rows * qph;
-    float m = 0.0f;
-    for (uint64_t i0 = 0; i0 < total; i0 += U * 256) {
+namespace {
+// Largest finite |element| (or m) a thread sees of the float4s of one head from
+// i0 on, the T threads of the workgroup taking U at a time; `first` ends the scan
+// with the first round in which any of them found one above 0.  Rows and columns
+// are stepped, not divided: eight 64-bit divisions a round outweighed its loads.
+template <int T, int U>
+__device__ __forceinline__ float head_amax(const float* __restrict__ src, uint32_t i0, uint32_t n_rows,
+                                           uint32_t qph, uint32_t row_len, bool first, float m) {
+    const uint32_t dr = T / qph, dc = T - dr * qph;  // T float4s further
+    uint64_t r = (i0 + threadIdx.x) / qph;
+    uint32_t c = i0 + threadIdx.x - (uint32_t)r * qph;
+    for (uint64_t at = i0; at < (uint64_t)n_rows * qph; at += U * T) {
         float4 x[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const uint64_t i = i0 + u * 256 + threadIdx.x;
-            const uint64_t ic = i < total ? i : i0;
-            const uint64_t r = ic / qph;
-            x[u] = *reinterpret_cast<const float4*>(src + r * row_len + 4 * (ic - r * qph));
+            // (past the end: row 0 again)
+            x[u] = *reinterpret_cast<const float4*>(src + (r < n_rows ? r : 0) * row_len + 4 * c);
+            r += dr;
+            c += dc;
+            if (c >= qph) {
+                c -= qph;
+                ++r;
+            }
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) m = finite_amax(x[u], m);
-        if (seed && __syncthreads_or(m > 0.0f)) break;  // uniform
+        if (first && __syncthreads_or(m > 0.0f)) break;  // uniform
     }
+    return m;
+}
+
+// The scale of the T threads' largest m, on thread 0.
+template <int T>
+__device__ __forceinline__ float workgroup_scale(float m, float* wmax) {
 #pragma unroll
     for (int o = 32; o >= 1; o >>= 1) {
         const float y = __shfl_xor(m, o, 64);
@@ -279,10 +285,48 @@ extern "C" __global__ __launch_bounds__(256) void eh_kv_e4m3_scales(
     }
     if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        for (uint32_t w = 1; w < blockDim.x / 64; ++w) m = wmax[w] > m ? wmax[w] : m;
-        (blockIdx.y ? v_scale : k_scale)[h] = e4m3_scale_of(m);
-    }
+    if (threadIdx.x == 0)
+        for (uint32_t w = 1; w < T / 64; ++w) m = wmax[w] > m ? wmax[w] : m;
+    return e4m3_scale_of(m);
+}
+}  // namespace
+
+// One workgroup per head.  Grid (n_kv, 2): y = 0 reads keys into k_scale,
+// y = 1 values into v_scale; 256 threads; head_dim % 4 == 0.
+extern "C" __global__ __launch_bounds__(256) void eh_kv_e4m3_scales(
+    const float* keys, const float* values, uint32_t n_rows, uint32_t row_len, uint32_t head_dim,
+    float* k_scale, float* v_scale) {
+    __shared__ float wmax[4];
+    const uint32_t h = blockIdx.x;
+    const float* src = (blockIdx.y ? values : keys) + (uint64_t)h * head_dim;
+    const uint32_t qph = head_dim / 4;  // float4s per head row
+    const float s = workgroup_scale<256>(
+        head_amax<256, 4>(src, 0, n_rows, qph, row_len, false, 0.0f), wmax);
+    if (threadIdx.x == 0) (blockIdx.y ? v_scale : k_scale)[h] = s;
+}
+
+// The first of the two launches for many rows: a lower bound of each scale from
+// the first rows that hold a finite nonzero element, for eh_kv_e4m3_scales_rows
+// to raise, and 1 only if no row holds one.  Grid (n_kv, 2), 1024 threads: a
+// head of zeros is walked to its end by this one workgroup, which is bound by
+// the loads it has in flight, 8 per thread from the second round on (4096 rows of
+// 8 heads of 128, one of them zeros: 47 us in all; 146 with 256 threads of 4
+// loads, 143 in one launch of those; 11 without such a head).  Counting the
+// workgroups that find nothing in the scale's own word, with the last one to
+// write the 1, took 108: 128 compare-exchanges of one word go one by one.
+extern "C" __global__ __launch_bounds__(1024) void eh_kv_e4m3_scales_seed(
+    const float* keys, const float* values, uint32_t n_rows, uint32_t row_len, uint32_t head_dim,
+    float* k_scale, float* v_scale) {
+    __shared__ float wmax[16];
+    const uint32_t h = blockIdx.x;
+    const float* src = (blockIdx.y ? values : keys) + (uint64_t)h * head_dim;
+    const uint32_t qph = head_dim / 4;
+    // (the host comes here with more than one round of rows)
+    float m = finite_amax(*reinterpret_cast<const float4*>(
+        src + (uint64_t)(threadIdx.x / qph) * row_len + 4 * (threadIdx.x % qph)), 0.0f);
+    if (!__syncthreads_or(m > 0.0f)) m = head_amax<1024, 8>(src, 1024, n_rows, qph, row_len, true, m);
+    const float s = workgroup_scale<1024>(m, wmax);
+    if (threadIdx.x == 0) (blockIdx.y ? v_scale : k_scale)[h] = s;
 }
 
 // Raises the seeded scales over all rows.  Scales of positive amax are
