@@ -906,3 +906,25 @@ def test_device_position_costs_by_its_length(dev):
             best = min(best, a.elapsed_time(b))
         took.append(best)
     assert took[1] < 3 * took[0], took
+
+
+@pytest.mark.parametrize("dtype,tokens", [(KvDataType.F32, 1 << 17), (KvDataType.BF16, 1 << 18)])
+def test_fused_step_in_a_page_beyond_4_gib(dev, dtype, tokens):
+    """One page of 8 GiB: the key that takes all the weight and the appended row lie
+    behind its first 4 GiB, and the row that a 32-bit offset would reach stays."""
+    n_head = n_kv = 64
+    hd, pos = 128, tokens // 2 + 4464
+    pool = torch.zeros((tokens, 2, n_kv * hd), device=dev, dtype=TD[dtype])
+    assert pool[:1].nbytes * (tokens // 2) == 1 << 32
+    g = torch.Generator(device=dev).manual_seed(5)
+    q = torch.randn((n_head, hd), device=dev, generator=g)
+    v = torch.randn((n_kv * hd,), device=dev, generator=g).to(TD[dtype])
+    pool[pos - 1, 0] = (10.0 * q).reshape(-1).to(TD[dtype])   # score 10 |q|^2 / sqrt(hd), about 113
+    pool[pos - 1, 1] = v
+    k_new = torch.zeros_like(v)
+    v_new = torch.full_like(v, 9.0)
+    out = torch.empty_like(q)
+    PagedAttention(0).append_flash_decoding(None, k_new, v_new, q, pool.reshape(-1), i32([0], dev), out, n_head,
+                                            n_kv, hd, tokens, pos, i32([pos], dev), dtype)
+    check_close(out.cpu().numpy(), v.float().cpu().numpy().reshape(n_head, hd), KvDataType.F32)
+    assert torch.equal(pool[pos, 1], v_new) and not pool[pos - tokens // 2].any()
