@@ -70,6 +70,8 @@ for case in json.load(sys.stdin):
     elt = 4 if dt == 0 else 2
     pages = -(-ctx_len // bt)
     qb, pool = batch * nh * hd * 4, pages * bt * 2 * nkv * hd * elt
+    if how.startswith("pool"):   # a pool of one page, less the named bytes
+        pool, how = bt * 2 * nkv * hd * elt - int(how.split()[1]), how.split()[2]
     if how == "plan":
         t, m, w = C.c_uint32(), C.c_uint32(), C.c_uint64()
         st = L.eh_decode_plan(dt, batch, nh, nkv, hd, bt, ctx_len, 0, C.byref(t), C.byref(m), C.byref(w))
@@ -135,3 +137,13 @@ def test_splits_near_the_largest(choose, how):
         assert tps <= largest and (name.startswith("eh_decode_split") or tps % tile == 0), case
         at_limit += tps > largest - 4 * tile
     assert at_limit > 20
+
+
+@pytest.mark.parametrize("how", ["fused", "host"])
+def test_a_pool_below_one_page_is_refused(choose, how):
+    """Masked keys read page 0, so a pool that holds no whole page launches nothing."""
+    shapes = [(dt, 1, 14, 2, hd, 16, 500) for dt in (0, 1, 3) for hd in (32, 64, 128)]
+    for st, launches in choose([(*s, f"pool 1 {how}") for s in shapes]):
+        assert st == 1 and launches == []
+    for st, launches in choose([(*s, f"pool 0 {how}") for s in shapes]):
+        assert st == 0 and launches

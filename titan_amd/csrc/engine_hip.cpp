@@ -1107,9 +1107,11 @@ static eh_status single_seq_attention(eh_context* c, eh_stream stream, uint32_t 
     eh_status st = validate_attention(kv_dtype, q_bytes, pool_bytes, bt_bytes, out_bytes, n_head,
                                       n_head_kv, head_dim, block_tokens, seq_tokens, query_pos);
     if (st) return st;
+    // (masked keys read page 0)
+    const uint64_t page_bytes = smul(block_tokens, 2, n_head_kv, head_dim, elt_bytes(kv_dtype));
+    if (pool_bytes < page_bytes) return invalid_size(page_bytes, pool_bytes);
     st = bind(c);
     if (st) return st;
-    const uint64_t page_bytes = smul(block_tokens, 2, n_head_kv, head_dim, elt_bytes(kv_dtype));
     decode_args a{};
     a.kv_dtype = kv_dtype;
     a.q = q;
