@@ -216,6 +216,27 @@ def test_layout_and_size_checks_before_any_hip_call():
     assert {k: tuple(v) for k, v in got.items()} == want
 
 
+@pytest.mark.parametrize("missing", [(), ("_cuda_getCurrentRawStream",), ("_cuda_getDevice",),
+                                     ("_cuda_getCurrentRawStream", "_cuda_getDevice")])
+def test_stream_handle_with_and_without_torchs_raw_functions(monkeypatch, missing):
+    """The current stream comes from torch's private raw-handle functions while torch
+    has them, else from its public interface; torch streams and handles pass through."""
+    import torch
+
+    from titan_amd.runtime import stream_handle
+
+    class Stream:
+        cuda_stream = 1234
+    monkeypatch.setattr(torch.cuda, "is_initialized", lambda: True)
+    monkeypatch.setattr(torch.cuda, "current_stream", Stream)
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: 3, raising=False)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda d: 5000 + d, raising=False)
+    for name in missing:
+        monkeypatch.delattr(torch._C, name)
+    assert stream_handle(None) == (1234 if missing else 5003)
+    assert stream_handle(Stream()) == 1234 and stream_handle(77) == 77
+
+
 def test_grid_workspace_bytes():
     """Workspace of a token-balanced decode at a caller-chosen grid: one
     (acc, m, l) partial per run and per sequence, 4 * (grid + batch) * n_head

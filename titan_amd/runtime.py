@@ -76,13 +76,16 @@ def ptr(x):
 
 def stream_handle(stream):
     """hipStream_t of a torch stream, a raw handle, or (None) torch's current
-    stream on its current device.  The latter is read as a raw handle:
+    stream on its current device.  The latter is read as a raw handle where
+    torch has the functions for it (they are not of its public interface):
     torch.cuda.current_stream() builds a Stream object, 3.1 us of a 13 us call
     where the handle takes 0.2."""
     if stream is None:
         import torch
-        if torch.cuda.is_initialized():
-            return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        device = getattr(torch._C, "_cuda_getDevice", None)
+        if raw is not None and device is not None and torch.cuda.is_initialized():
+            return raw(device())
         return torch.cuda.current_stream().cuda_stream
     if isinstance(stream, int):
         return stream
