@@ -85,14 +85,17 @@ for case in json.load(sys.stdin):
     else:                   # host position ctx_len - 1
         st = L.eh_flash_decoding(ctx, None, dt, P, qb, P, pool, P, pages * 4, P, qb, nh, nkv, hd, bt,
                                  ctx_len, ctx_len - 1, 1, None)
-    out.append((st, launches()))
+    name = C.create_string_buffer(64)
+    assert L.eh_decode_kernel_name(dt, nh, nkv, hd, bt, name, 64) == 0
+    out.append((st, launches(), name.value.decode()))
 print(json.dumps(out))
 """
 
 
 @pytest.fixture(scope="module")
 def choose(tmp_path_factory):
-    """cases [(dtype, batch, n_head, n_kv, head_dim, block_tokens, context, how)] -> [(status, launches)]."""
+    """cases [(dtype, batch, n_head, n_kv, head_dim, block_tokens, context, how)] -> [(status, launches,
+    name of the batched split kernel)]."""
     d = tmp_path_factory.mktemp("hip")
     (d / "hip.c").write_text(_HIP)
     so = str(d / "hip.so")
@@ -125,7 +128,7 @@ def test_splits_near_the_largest(choose, how):
                             cases += [(dt, b, nh, nkv, hd, bt, ctx, how)
                                       for b in ((2, 16, 32, 128, 256) if how == "plan" else (1,))]
     at_limit = 0
-    for case, (st, launches) in zip(cases, choose(cases)):
+    for case, (st, launches, _) in zip(cases, choose(cases)):
         assert st == 0, case
         name, _, tps, splits = launches[0]
         if not name.startswith(("eh_decode_rows", "eh_decode_split")):
@@ -143,7 +146,15 @@ def test_splits_near_the_largest(choose, how):
 def test_a_pool_below_one_page_is_refused(choose, how):
     """Masked keys read page 0, so a pool that holds no whole page launches nothing."""
     shapes = [(dt, 1, 14, 2, hd, 16, 500) for dt in (0, 1, 3) for hd in (32, 64, 128)]
-    for st, launches in choose([(*s, f"pool 1 {how}") for s in shapes]):
+    for st, launches, _ in choose([(*s, f"pool 1 {how}") for s in shapes]):
         assert st == 1 and launches == []
-    for st, launches in choose([(*s, f"pool 0 {how}") for s in shapes]):
+    for st, launches, _ in choose([(*s, f"pool 0 {how}") for s in shapes]):
         assert st == 0 and launches
+
+
+def test_kernel_name_is_the_batched_launch(choose):
+    """eh_decode_kernel_name names what a batch launches."""
+    cases = [(dt, b, nh, nkv, hd, bt, 1000, "plan") for dt in (0, 1, 3) for hd in (32, 64, 128)
+             for nh, nkv in HEADS for bt in (4, 8, 16, 24) for b in (2, 16)]
+    for case, (st, launches, name) in zip(cases, choose(cases)):
+        assert st == 0 and launches[0][0] == name, case

@@ -1313,7 +1313,8 @@ eh_status eh_decode_kernel_name(uint32_t kv_dtype, uint32_t n_head, uint32_t n_h
     if (block_tokens < 1) return fail(EH_INVALID_ARGS, "block_tokens");
     const char* dn = kv_dtype == EH_KV_FP8 ? "fp8" : dt_name(kv_dtype);
     if (!dn) return fail(EH_UNSUPPORTED, "kv_dtype");
-    const decode_kernel dk = pick_decode_kernel(kv_dtype, head_dim, n_head, n_head_kv, block_tokens, 1);
+    // (of a batch: one sequence of f32 at head_dim 128 runs the row kernels)
+    const decode_kernel dk = pick_decode_kernel(kv_dtype, head_dim, n_head, n_head_kv, block_tokens, 2);
     const tiles_cfg tc = pick_tiles(kv_dtype, head_dim, n_head, n_head_kv, block_tokens, 1);
     char name[64];
     if (kv_dtype == EH_KV_FP8 && !tc.ok) return fail(EH_UNSUPPORTED, "E4M3 shape");
