@@ -829,7 +829,8 @@ def test_row_kernels_heads_of_any_magnitude(dev, dtype, hd):
 
 
 LONG_TABLES = [  # (n_head, n_kv, head_dim, block_tokens, table entries)
-    (32, 32, 128, 16, 8192), (14, 2, 64, 8, 8192), (12, 3, 128, 4, 20000), (16, 1, 64, 32, 3000)]
+    (32, 32, 128, 16, 8192), (14, 2, 64, 8, 8192), (12, 3, 128, 4, 20000), (16, 1, 64, 32, 3000),
+    (8, 2, 32, 16, 8192), (6, 3, 128, 24, 3000)]   # (the per-token kernel)
 
 
 @pytest.mark.parametrize("dtype", [KvDataType.F32, KvDataType.F16, KvDataType.BF16])

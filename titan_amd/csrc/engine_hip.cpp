@@ -249,8 +249,8 @@ struct decode_kernel {
     uint32_t g = 1;       // head-major: compiled head-group width
     uint32_t chunks = 1;  // workgroups per (split, kv head, sequence)
     uint64_t chunk = 1;   // a split is a multiple of this many tokens
-    uint64_t round = 1;   // tokens one pass of the workgroup's waves takes (planned splits, and
-                          // the row kernels' own ones: live_tps in decode_len.h)
+    uint64_t round = 1;   // tokens one pass of the workgroup's waves takes, a power of two (planned
+                          // splits, and those the kernels cut themselves: live_tps in decode_len.h)
     uint64_t units = 1;   // workgroups per (split, sequence)
 };
 
@@ -321,26 +321,24 @@ eh_status run_decode(eh_context* c, eh_stream stream, const decode_args& a) {
     const hipModule_t mod = c->mod_decode[dt_index(a.kv_dtype)];
     const dim3 grid = dk.rows ? dim3(a.batch, a.n_head_kv * dk.chunks, a.max_splits)
                               : dim3(a.max_splits, a.n_head_kv * dk.chunks, a.batch);
-    // device position: contexts from which the row kernels cut shorter splits (live_tps)
+    // device position: contexts from which the kernels cut shorter splits (live_tps)
+    const uint32_t round_log2 = (uint32_t)log2_exact(dk.round);
     const uint32_t shorter =
-        dk.rows && a.lens_mode == 1 && a.tps > dk.round
+        a.lens_mode == 1 && a.tps > dk.round
             ? (uint32_t)std::min<uint64_t>((uint64_t)a.max_splits * (a.tps - dk.round) + 1, 0xFFFFFFFFu)
             : 0u;
-    auto split = [&](hipModule_t m, auto... more) {
-        return launch(c, m, name, grid, dim3(kDecodeThreads), stream, a.q, (const uint8_t*)a.pool, a.bt,
-                      a.bt_stride, a.lens_ptr, a.lens_mode, a.seq_tokens, a.query_pos, a.causal, a.out,
-                      a.part_acc, a.part_ml, a.n_head, a.n_head_kv, a.block_tokens, bt_shift, a.tps,
-                      a.max_splits, scale_log2, a.n_blocks, (const uint8_t*)a.new_k,
-                      (const uint8_t*)a.new_v, more...);
-    };
-    eh_status st = dk.rows ? split(c->mod_rows, shorter) : split(mod);
+    eh_status st = launch(c, dk.rows ? c->mod_rows : mod, name, grid, dim3(kDecodeThreads), stream,
+                          a.q, (const uint8_t*)a.pool, a.bt, a.bt_stride, a.lens_ptr, a.lens_mode,
+                          a.seq_tokens, a.query_pos, a.causal, a.out, a.part_acc, a.part_ml, a.n_head,
+                          a.n_head_kv, a.block_tokens, bt_shift, a.tps, a.max_splits, scale_log2,
+                          a.n_blocks, (const uint8_t*)a.new_k, (const uint8_t*)a.new_v, round_log2, shorter);
     if (st != EH_OK || a.max_splits <= 1) return st;
     return launch(c, mod, "eh_decode_merge",
                   dim3((uint32_t)div_ceil((uint64_t)a.n_head * a.head_dim, 64), a.batch), dim3(256),
                   stream,
                   (const float*)a.part_acc, (const float*)a.part_ml, a.out, a.lens_ptr, a.lens_mode,
                   a.seq_tokens, a.query_pos, a.causal, a.n_head, a.head_dim, a.tps, a.max_splits,
-                  (uint32_t)std::max(log2_exact(dk.round), 0), shorter);
+                  round_log2, shorter);
 }
 
 // ---- token-balanced decode (eh_decode_tiles_*, paged_decode_tiles.hip)

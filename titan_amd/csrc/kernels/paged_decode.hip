@@ -146,7 +146,7 @@ __device__ __forceinline__ void decode_split(
     float* __restrict__ part_acc, float* __restrict__ part_ml, uint32_t n_head,
     uint32_t n_head_kv, uint32_t block_tokens, int bt_shift, uint32_t tps, uint32_t max_splits,
     float scale_log2, uint64_t n_blocks, const uint8_t* __restrict__ new_k,
-    const uint8_t* __restrict__ new_v) {
+    const uint8_t* __restrict__ new_v, uint32_t round_log2, uint32_t shorter) {
     constexpr int ELT = dt_info<DT>::bytes;
     constexpr int EPL = (16 / ELT) < HD ? (16 / ELT) : HD;  // elements per lane
     constexpr int LPT = HD / EPL;                            // lanes per token row
@@ -170,7 +170,7 @@ __device__ __forceinline__ void decode_split(
     const uint32_t b = blockIdx.z;
     const uint32_t qh0 = hk * group + hc * G;
 
-    const uint32_t t0 = split * tps;
+    uint32_t t0 = split * tps;
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int grp = lane / LPT;
@@ -191,13 +191,17 @@ __device__ __forceinline__ void decode_split(
     // known: with a device position that length is one more memory round
     // trip.  Entries past the length are staged and never read; the host's
     // bound on tokens per split keeps a whole range's slice inside BT_SLICE.
-    const uint32_t pg0 = page_of(t0);
-    const uint32_t t_end = t0 > 0xFFFFFFFFu - tps ? 0xFFFFFFFFu : t0 + tps;  // >= every t1
-    const uint32_t npg = page_of(t_end - 1) - pg0 + 1;
-    for (uint32_t i = threadIdx.x; i < npg && i < BT_SLICE; i += NW * 64) {
-        const uint32_t pg = pg0 + i;
-        s_bt[i] = pg < bt_stride ? bt_row[pg] : 0xFFFFFFFFu;
-    }
+    uint32_t pg0;
+    auto stage = [&] {
+        pg0 = page_of(t0);
+        const uint32_t t_end = t0 > 0xFFFFFFFFu - tps ? 0xFFFFFFFFu : t0 + tps;  // >= every t1
+        const uint32_t npg = page_of(t_end - 1) - pg0 + 1;
+        for (uint32_t i = threadIdx.x; i < npg && i < BT_SLICE; i += NW * 64) {
+            const uint32_t pg = pg0 + i;
+            s_bt[i] = pg < bt_stride ? bt_row[pg] : 0xFFFFFFFFu;
+        }
+    };
+    stage();
 
     // Query slice of every head in this chunk, pre-scaled into the log2
     // domain.  Loads are unconditional (heads past the group re-read the last
@@ -222,6 +226,12 @@ __device__ __forceinline__ void decode_split(
     }
 
     const uint32_t n = live_tokens(L, b);
+    const uint32_t cut = live_tps(n, tps, max_splits, round_log2, shorter);
+    if (cut != tps) {  // uniform: a device position far below the table's capacity
+        tps = cut;
+        t0 = split * tps;
+        if (t0 < n) stage();  // (each thread over its own entries)
+    }
     if (t0 >= n) {  // uniform over the workgroup
         // No live tokens at all: the output is zero (forward_cpu.rs:436-439).
         if (n == 0 && split == 0)
@@ -467,11 +477,11 @@ extern "C" __global__ __launch_bounds__(256) void eh_decode_merge(
         uint32_t causal, float* out, float* part_acc, float* part_ml, uint32_t n_head,          \
         uint32_t n_head_kv, uint32_t block_tokens, int bt_shift, uint32_t tps,                  \
         uint32_t max_splits, float scale_log2, uint64_t n_blocks, const uint8_t* new_k,         \
-        const uint8_t* new_v) {                                                                 \
+        const uint8_t* new_v, uint32_t round_log2, uint32_t shorter) {                          \
         const len_src L{lens_ptr, lens_mode, seq_tokens, query_pos, causal};                    \
         decode_split<DT, HD, G>(q, pool, bt, bt_stride, L, out, part_acc, part_ml, n_head,      \
                                 n_head_kv, block_tokens, bt_shift, tps, max_splits, scale_log2, \
-                                n_blocks, new_k, new_v);                                        \
+                                n_blocks, new_k, new_v, round_log2, shorter);                   \
     }
 
 #define EH_DECODE_G(DTN, DT, HD) \
