@@ -280,10 +280,11 @@ eh_status eh_decode_plan(uint32_t kv_dtype, uint32_t batch, uint32_t n_head, uin
  * every run plus one per sequence, or UINT64_MAX where that does not fit
  * 64 bits (no reference counterpart). */
 uint64_t eh_decode_grid_workspace_bytes(uint32_t grid, uint32_t batch, uint32_t n_head);
-/* Name of the split kernel eh_paged_decode_batched launches for a shape and two
- * or more sequences under a plan without a hint (diagnostics and profiling; no
- * reference counterpart).  One sequence runs the same, except f32 at head_dim 128:
- * eh_decode_rows_f32_hd128. */
+/* Name of the split kernel eh_paged_decode_batched launches for a shape and a few
+ * sequences of many thousand tokens under a plan without a hint (diagnostics and
+ * profiling; no reference counterpart).  The length and the number of sequences
+ * count for pages under 8 tokens and for f32 pages only: one sequence at head_dim
+ * 128 runs eh_decode_rows_f32_hd128. */
 eh_status eh_decode_kernel_name(uint32_t kv_dtype, uint32_t n_head, uint32_t n_head_kv,
                                 uint32_t head_dim, uint32_t block_tokens, char* buf, uint64_t size);
 /* q/out [batch, n_head, head_dim] f32; block_tables [batch, bt_stride] u32;

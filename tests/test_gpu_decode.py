@@ -655,7 +655,9 @@ def test_graph_replay_split_count_follows_device_position(dev):
 
 
 ROW_SHAPES = [  # (n_head, n_kv, head_dim, block_tokens)
-    (14, 2, 64, 16), (17, 1, 128, 8), (32, 2, 64, 64), (9, 3, 128, 4), (5, 5, 64, 1)]
+    (14, 2, 64, 16), (17, 1, 128, 8), (32, 2, 64, 64), (9, 3, 128, 4), (5, 5, 64, 1),
+    (20, 2, 64, 4), (7, 1, 128, 1), (15, 3, 64, 2), (32, 1, 128, 2),   # pages under 8 tokens: 5 heads and more
+    (8, 4, 64, 16), (3, 3, 64, 8)]   # f32: 1 or 2 heads, 40 and 30 kv heads in the batch of 10
 
 
 @pytest.mark.parametrize("dtype", [KvDataType.F32, KvDataType.F16, KvDataType.BF16])
@@ -830,7 +832,7 @@ def test_row_kernels_heads_of_any_magnitude(dev, dtype, hd):
 
 LONG_TABLES = [  # (n_head, n_kv, head_dim, block_tokens, table entries)
     (32, 32, 128, 16, 8192), (14, 2, 64, 8, 8192), (12, 3, 128, 4, 20000), (16, 1, 64, 32, 3000),
-    (8, 2, 32, 16, 8192), (6, 3, 128, 24, 3000)]   # (the per-token kernel)
+    (14, 2, 64, 4, 8192), (8, 2, 32, 16, 8192), (6, 3, 128, 24, 3000)]   # (the last two: the per-token kernel)
 
 
 @pytest.mark.parametrize("dtype", [KvDataType.F32, KvDataType.F16, KvDataType.BF16])

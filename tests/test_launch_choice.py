@@ -154,7 +154,38 @@ def test_a_pool_below_one_page_is_refused(choose, how):
 
 def test_kernel_name_is_the_batched_launch(choose):
     """eh_decode_kernel_name names what a batch launches."""
-    cases = [(dt, b, nh, nkv, hd, bt, 1000, "plan") for dt in (0, 1, 3) for hd in (32, 64, 128)
-             for nh, nkv in HEADS for bt in (4, 8, 16, 24) for b in (2, 16)]
+    cases = [(dt, b, nh, nkv, hd, bt, 32768, "plan") for dt in (0, 1, 3) for hd in (32, 64, 128)
+             for nh, nkv in HEADS for bt in (4, 8, 16, 24) for b in (2, 16)
+             if b == 2 or (bt >= 8 and dt != 0)]   # (the length and number count for the others)
     for case, (st, launches, name) in zip(cases, choose(cases)):
         assert st == 0 and launches[0][0] == name, case
+
+
+def test_kernel_by_page_size_and_heads(choose):
+    """Pages under 8 tokens and up to 4 q heads per kv head: the per-token kernel from
+    98304 tokens over the batch's kv heads on (196608 at 3 and 4 heads) and for fused
+    steps up to 384; f32 batches at head_dim 64 with 1 or 2: from 131072 on; and back
+    to the row kernels where the per-token kernel's largest split (992 tokens of
+    pages of one) is too short."""
+    def kernels(cases):
+        return [launches[0][0].split("_hd")[0] for st, launches, _ in choose(cases) if st == 0]
+    small, want = [], []
+    for dt in (1, 3):
+        for hd in (64, 128):
+            for bt in (1, 2, 4):
+                for g in (1, 2, 3, 4, 5, 16):
+                    for ctx in (384, 23040, 25600, 46080, 51200):   # 4 kv heads; whole splits of either
+                        small.append((dt, 2, 2 * g, 2, hd, bt, ctx, "plan"))
+                        split = g <= 4 and 4 * ctx >= (98304 if g <= 2 else 196608)
+                        want.append("eh_decode_" + ("split" if split else "rows") + ("_f16" if dt == 1 else "_bf16"))
+    assert kernels(small) == want
+    step = [(1, 1, 3 * g, 3, 64, 4, ctx, "fused") for g in (1, 2, 4, 5) for ctx in (384, 512, 49152, 81920)]
+    names = ["split", "rows", "split", "split"] * 2 + ["split", "rows", "rows", "split"] + ["rows"] * 4
+    assert kernels(step) == [f"eh_decode_{n}_f16" for n in names]
+    f32 = [(0, b, nkv * g, nkv, 64, 16, ctx, "plan") for b, nkv, ctx in ((1, 64, 4096), (2, 32, 1024), (2, 32, 3072),
+                                                                         (16, 4, 1792), (16, 4, 2304)) for g in (1, 2, 3)]
+    want = ["eh_decode_" + ("split" if c[1] > 1 and c[1] * c[3] * c[6] >= 131072 and c[2] <= 2 * c[3] else "rows") + "_f32"
+            for c in f32]
+    assert kernels(f32) == want
+    far = [(1, 1, 3, 3, 64, 1, ctx, how) for ctx in (256 * 992, 256 * 992 + 1) for how in ("fused", "host", "plan")]
+    assert kernels(far) == ["eh_decode_split_f16"] * 3 + ["eh_decode_rows_f16"] * 3

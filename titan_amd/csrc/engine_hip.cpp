@@ -236,9 +236,22 @@ uint64_t chunk_tokens(uint32_t kv_dtype, uint64_t head_dim) {
 //     pages (f32: of at least 8 tokens); MFMA, up to 16 q heads of a kv head per
 //     workgroup, K read along its rows;
 //   head-major (eh_decode_split_*, paged_decode.hip): everything else, splits
-//     that are no whole tiles of the former, and f32 batches at head_dim 128,
-//     which HBM bounds in either (16 sequences of 64 .. 4096 tokens, 32/8 heads:
-//     74 us in both).
+//     that are no whole tiles of the former, f32 batches at head_dim 128, which
+//     HBM bounds in either (16 sequences of 64 .. 4096 tokens, 32/8 heads: 74 us in
+//     both), and two cases where it is the faster one:
+//     pages under 8 tokens at up to 4 q heads per kv head -- the row kernels look
+//     every key's page up and its row waits for that, which shows once the chip is
+//     full (from 98304 tokens over the batch's kv heads on, 196608 at 3 and 4 q
+//     heads) and in fused steps of up to 384 tokens.  Pages of 2, rows / head-major,
+//     us: a fused step at 12000 tokens, f16, 32/32 heads of 64 58.8 / 25.1, 16 ragged
+//     sequences up to 12000, bf16, 128/32 heads 380 / 190, 4 of 2048, f16, 16/16 heads
+//     1.2 of head-major, 4 of 1024 1.1, a fused step of 8, 32/32 heads of 128 10.2 /
+//     5.0, of 256 1.5 of it, of 1024 1.1; from 5 q heads on the matrix work outweighs
+//     it (16 of 8192, 14/2 heads of 64 29 / 40);
+//     f32 batches at head_dim 64, 1 or 2 q heads per kv head, from 131072 tokens over
+//     the batch's kv heads on -- a key's row serves too few heads (16 ragged sequences
+//     up to 2048 tokens, 32/32 heads 71 / 61, up to 1024, 16/16 heads 25 / 20; 4 of
+//     4096, 4/4 heads 0.97 of head-major, of 1024 0.9).
 // Measured, before / with the row kernels, us: 16 sequences of 64 .. 4096
 // tokens at 14/2 heads of 64 f16 20.2 / 11.0, bf16 21.0 / 11.3, f32 22.0 / 15.1;
 // 24/3 heads 33.8 / 14.2; one sequence of 8191 tokens, 32/8 heads of 128, f16
@@ -254,17 +267,24 @@ struct decode_kernel {
     uint64_t units = 1;   // workgroups per (split, sequence)
 };
 
-// tps: the split the caller asks for (0: still to be planned).
+// ctx: tokens a sequence may have; fused: with the append; tps: the split the caller asks for (0: still to
+// be planned, `least` tokens or more, which rules out a kernel whose largest split
+// is shorter).
 decode_kernel pick_decode_kernel(uint32_t kv_dtype, uint64_t head_dim, uint64_t n_head,
                                  uint64_t n_head_kv, uint64_t block_tokens, uint64_t batch,
-                                 uint64_t tps = 0) {
+                                 uint64_t ctx, bool fused, uint64_t tps, uint64_t least) {
     decode_kernel k;
     const uint32_t group = (uint32_t)(n_head / n_head_kv);
     const uint64_t tile = kv_dtype == EH_KV_F32 ? 16 : 32;  // mirrors TK in paged_rows.hip
     const int shift = log2_exact(block_tokens);
     const bool f32 = kv_dtype == EH_KV_F32;
+    const uint64_t work = smul(batch, n_head_kv, ctx);
+    const bool per_token =
+        (shift < 3 ? group <= 4 && (work >= (group <= 2 ? 98304u : 196608u) || (fused && ctx <= 384))
+                   : f32 && head_dim == 64 && group <= 2 && batch > 1 && work >= 131072) &&
+        std::max(tps, least) <= max_tps(block_tokens, chunk_tokens(kv_dtype, head_dim), false);
     if ((head_dim == 64 || head_dim == 128) && shift >= (f32 ? 3 : 0) && tps % tile == 0 &&
-        !(f32 && head_dim == 128 && batch > 1)) {
+        !(f32 && head_dim == 128 && batch > 1) && !per_token) {
         k.rows = true;
         k.chunks = (group + 15) / 16;
         k.chunk = tile;
@@ -305,7 +325,8 @@ eh_status run_decode(eh_context* c, eh_stream stream, const decode_args& a) {
     if (!supported_hd(a.kv_dtype, a.head_dim)) return fail(EH_UNSUPPORTED, "head_dim", 256, a.head_dim);
     if (a.max_splits > kMaxSplits) return invalid_size(kMaxSplits, a.max_splits, "max_splits");
     const decode_kernel dk =
-        pick_decode_kernel(a.kv_dtype, a.head_dim, a.n_head, a.n_head_kv, a.block_tokens, a.batch, a.tps);
+        pick_decode_kernel(a.kv_dtype, a.head_dim, a.n_head, a.n_head_kv, a.block_tokens, a.batch,
+                           (uint64_t)a.tps * a.max_splits, a.new_k != nullptr, a.tps, 0);
     char name[64];
     if (dk.rows)
         std::snprintf(name, sizeof name, "eh_decode_rows_%s_hd%u%s%s", dn, a.head_dim,
@@ -1132,8 +1153,8 @@ static eh_status single_seq_attention(eh_context* c, eh_stream stream, uint32_t 
     // device, so size the grid for everything the block table can address.
     uint64_t cap = seq_tokens;
     if (pos_ptr) cap = std::max<uint64_t>(cap, (uint64_t)a.bt_stride * block_tokens);
-    const decode_kernel dk =
-        pick_decode_kernel(kv_dtype, head_dim, n_head, n_head_kv, block_tokens, 1);
+    const decode_kernel dk = pick_decode_kernel(kv_dtype, head_dim, n_head, n_head_kv, block_tokens, 1,
+                                                cap, new_k != nullptr, 0, div_ceil(cap, kMaxSplits));
     const uint64_t chunk = dk.chunk;
     const uint64_t most = max_tps(block_tokens, chunk, dk.rows);
     // One sequence: a quarter of the workgroups per kv head for the row kernels,
@@ -1287,7 +1308,8 @@ eh_status eh_decode_plan(uint32_t kv_dtype, uint32_t batch, uint32_t n_head, uin
         if (workspace_bytes) *workspace_bytes = tiles_ws_bytes(grid, batch, n_head);
         return EH_OK;
     }
-    const decode_kernel dk = pick_decode_kernel(kv_dtype, head_dim, n_head, n_head_kv, block_tokens, batch);
+    const decode_kernel dk = pick_decode_kernel(kv_dtype, head_dim, n_head, n_head_kv, block_tokens, batch,
+                                                max_ctx, false, 0, std::max<uint64_t>(hint, div_ceil(max_ctx, kMaxSplits)));
     // The row kernels balance ragged lengths with twice the workgroups (8
     // sequences of 500 .. 12000 tokens, 56/8 heads of 64: 37.9 us at 1024, 37.3 at
     // 2048, 42.3 at 4096), but none under 128 tokens, whose merge costs more than
@@ -1295,9 +1317,10 @@ eh_status eh_decode_plan(uint32_t kv_dtype, uint32_t batch, uint32_t n_head, uin
     uint64_t tps = hint      ? div_ceil(hint, dk.chunk) * dk.chunk
                    : dk.rows ? std::max<uint64_t>(auto_tps(batch, dk, max_ctx, block_tokens, 2048), 128)
                              : auto_tps(batch, dk, max_ctx, block_tokens);
-    while (div_ceil(max_ctx ? max_ctx : 1, tps) > kMaxSplits) tps *= 2;
-    if (tps > max_tps(block_tokens, dk.chunk, dk.rows))
-        return invalid_size(max_tps(block_tokens, dk.chunk, dk.rows), tps, "tokens_per_split");
+    const uint64_t most = max_tps(block_tokens, dk.chunk, dk.rows);
+    while (div_ceil(max_ctx ? max_ctx : 1, tps) > kMaxSplits)
+        tps = tps < most ? std::min(2 * tps, most) : 2 * tps;
+    if (tps > most) return invalid_size(most, tps, "tokens_per_split");
     const uint32_t ms = (uint32_t)div_ceil(max_ctx ? max_ctx : 1, tps);
     if (tokens_per_split) *tokens_per_split = (uint32_t)tps;
     if (max_splits) *max_splits = ms;
@@ -1311,8 +1334,9 @@ eh_status eh_decode_kernel_name(uint32_t kv_dtype, uint32_t n_head, uint32_t n_h
     if (block_tokens < 1) return fail(EH_INVALID_ARGS, "block_tokens");
     const char* dn = kv_dtype == EH_KV_FP8 ? "fp8" : dt_name(kv_dtype);
     if (!dn) return fail(EH_UNSUPPORTED, "kv_dtype");
-    // (of a batch: one sequence of f32 at head_dim 128 runs the row kernels)
-    const decode_kernel dk = pick_decode_kernel(kv_dtype, head_dim, n_head, n_head_kv, block_tokens, 2);
+    // (two sequences of 32768 tokens)
+    const decode_kernel dk = pick_decode_kernel(kv_dtype, head_dim, n_head, n_head_kv, block_tokens, 2,
+                                                32768, false, 0, 0);
     const tiles_cfg tc = pick_tiles(kv_dtype, head_dim, n_head, n_head_kv, block_tokens, 1);
     char name[64];
     if (kv_dtype == EH_KV_FP8 && !tc.ok) return fail(EH_UNSUPPORTED, "E4M3 shape");

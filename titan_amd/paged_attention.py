@@ -110,8 +110,8 @@ class PagedAttention:
 
     @staticmethod
     def kernel_name(n_head, n_head_kv, head_dim, block_tokens, kv_dtype=KvDataType.F16):
-        """Split kernel decode_batched launches for this shape and two or more
-        sequences, planned without a hint."""
+        """Split kernel decode_batched launches for this shape and a few sequences
+        of many thousand tokens, planned without a hint."""
         buf_ = C.create_string_buffer(64)
         check(_lib.load().eh_decode_kernel_name(int(kv_dtype), int(n_head), int(n_head_kv),
                                                 int(head_dim), int(block_tokens), buf_, 64))
