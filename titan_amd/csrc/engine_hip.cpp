@@ -1312,11 +1312,26 @@ eh_status eh_decode_plan(uint32_t kv_dtype, uint32_t batch, uint32_t n_head, uin
                                                 max_ctx, false, 0, std::max<uint64_t>(hint, div_ceil(max_ctx, kMaxSplits)));
     // The row kernels balance ragged lengths with twice the workgroups (8
     // sequences of 500 .. 12000 tokens, 56/8 heads of 64: 37.9 us at 1024, 37.3 at
-    // 2048, 42.3 at 4096), but none under 128 tokens, whose merge costs more than
-    // it spreads (f32, 14/2 heads of 64: 15.1 us at 128, 17.6 at 64).
-    uint64_t tps = hint      ? div_ceil(hint, dk.chunk) * dk.chunk
-                   : dk.rows ? std::max<uint64_t>(auto_tps(batch, dk, max_ctx, block_tokens, 2048), 128)
-                             : auto_tps(batch, dk, max_ctx, block_tokens);
+    // 2048, 42.3 at 4096).  That many pay once they hold 384 tokens each (f32 256);
+    // shorter splits are for filling the chip alone, 512 workgroups, and end at 128
+    // tokens and 1/32 of the context (f32 1/64), where their merge costs more than
+    // they spread.  16 sequences, f16, by 2048 workgroups / so, us: 14/2 heads of 64
+    // at 6000 tokens 17.9 / 14.7, 1/1 heads at 12000 18.1 / 14.6, 12/3 heads of 128
+    // at 2048 17.0 / 15.5; 4 sequences of 2048, 32/32 heads of 128, 32.6 / 27.1; f32,
+    // 16 ragged up to 12000, 1/1 heads of 64, 22.3 / 19.4.
+    uint64_t tps;
+    if (hint) {
+        tps = div_ceil(hint, dk.chunk) * dk.chunk;
+    } else {
+        tps = auto_tps(batch, dk, max_ctx, block_tokens, dk.rows ? 2048 : 1024);
+        if (dk.rows) {
+            const bool f32 = kv_dtype == EH_KV_F32;
+            const uint64_t fill = std::max(div_ceil(smul(batch, dk.units, max_ctx), 512),
+                                           div_ceil(max_ctx, f32 ? 64 : 32));
+            const uint64_t least = std::min<uint64_t>(std::max<uint64_t>(fill, 128), f32 ? 256 : 384);
+            tps = std::max(tps, div_ceil(least, dk.round) * dk.round);
+        }
+    }
     const uint64_t most = max_tps(block_tokens, dk.chunk, dk.rows);
     while (div_ceil(max_ctx ? max_ctx : 1, tps) > kMaxSplits)
         tps = tps < most ? std::min(2 * tps, most) : 2 * tps;
