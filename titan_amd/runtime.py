@@ -82,10 +82,11 @@ def stream_handle(stream):
     where the handle takes 0.2."""
     if stream is None:
         import torch
-        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-        device = getattr(torch._C, "_cuda_getDevice", None)
-        if raw is not None and device is not None and torch.cuda.is_initialized():
-            return raw(device())
+        if torch.cuda.is_initialized():
+            try:
+                return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+            except AttributeError:
+                pass
         return torch.cuda.current_stream().cuda_stream
     if isinstance(stream, int):
         return stream
