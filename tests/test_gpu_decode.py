@@ -144,7 +144,7 @@ def test_batched_decode_ragged(dev, dtype):
         check_close(out.cpu().numpy(), ref, dtype)
 
 
-SHAPES = [  # (n_head, n_kv, head_dim, block_tokens): every slot-major head grouping,
+SHAPES = [  # (n_head, n_kv, head_dim, block_tokens): q heads per kv head 1 to 32,
     (8, 8, 128, 16), (16, 8, 64, 16), (6, 2, 64, 16), (4, 1, 128, 32), (8, 1, 128, 16),
     (14, 2, 128, 16), (24, 2, 128, 8), (32, 1, 64, 16), (64, 2, 128, 16), (10, 2, 64, 16),
     (12, 4, 128, 1), (12, 3, 128, 16), (12, 4, 128, 6), (8, 2, 32, 16)]  # ... and fallbacks

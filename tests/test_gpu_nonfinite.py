@@ -9,7 +9,7 @@ such a V row (0 * NaN = NaN) would fail.  The paths covered:
     the fused append, including appends that open a new tile (old length 0,
     16, 32, ...), whose tile's other rows are not written;
   * the same over E4M3 pages;
-  * the fixed-split and slot-major kernels of one sequence, with host and
+  * the fixed-split kernels of one sequence (f32 and 16-bit), with host and
     device positions, the fused append onto a new page, and invalid table
     entries inside the attended range (their stand-in, page 0, is NaN);
   * the single-pass decode of one sequence and the batched fixed-split
@@ -211,7 +211,7 @@ def test_e4m3_decode_and_step(dev):
                                       (KvDataType.F16, 128)], ids=["f32-64", "f16-64", "f16-128"])
 def test_single_sequence_decode(dev, dtype, hd):
     """Split-K decode of one sequence (f32: the fixed-split kernel, config
-    1's; f16: the slot-major kernel), 14/2 heads, pages of 16, NaN-tailed:
+    1's; f16 alike), 14/2 heads, pages of 16, NaN-tailed:
     host position, device position under a larger grid bound, and (f32,
     which has it) the fused append onto a new page (position 512, the first
     row of its page, not written before the launch)."""

@@ -592,6 +592,10 @@ bool prefill_pingpong(const prefill_args& a) {
 //   bf16 94 / 26, 117 / 59, 25 / 26, 108-138 / 113-123;  13 / 9.8, 36 / 20, -, 23-57 / 28-44
 //   E4M3 85 / 23, 105 / 47, 22 / 24, 98-124 / 88-96;  10 / 9.7, 32 / 21, -, 20-52 / 28-45
 //   f32 (512 tokens) 142 / 29, 266 / 73, 62 / 42, 205-394 / 123-175;  14 / 9.8, 140 / 37, -, 46-266 / 42-105
+// and at head_dim 64, 32/8 heads, 512 (f32 1024) workgroups, on 2000, 500, 100 and 0
+// tokens, where the key-split kernels are ahead as well:
+//   f16 55 / 30, 22 / 16, 14 / 13, 10.7 / 10.3;  bf16 69 / 37, 28 / 18, 17 / 13, 13 / 10;
+//   E4M3 57 / 29, 23 / 16, 14 / 13, 11.2 / 10.4;  f32 307 / 173, 107 / 70, 57 / 40, 40 / 31
 constexpr uint32_t kRowsRows = 32;  // query rows per workgroup, mirrors ROWS
 bool prefill_few_rows(const prefill_args& a) {
     if (log2_exact(a.block_tokens) < 3) return false;

@@ -206,7 +206,8 @@ __device__ __forceinline__ void append_e4m3_body(
 }  // namespace
 
 // Quantising append: f32 keys/values [n_tokens, row_len] -> E4M3 page rows,
-// 4 elements (one u32 of codes) per thread; addressing as eh_append_kv_c*.
+// 4 elements (one u32 of codes) per thread, from WIDE_UNITS on 16 or 8 of one
+// token's row; addressing as eh_append_kv_c*.
 extern "C" __global__ __launch_bounds__(256) void eh_append_kv_e4m3(
     const float* keys, const float* values, const uint32_t* bt, uint32_t bt_stride, uint8_t* pool,
     uint32_t n_tokens, uint32_t start, const uint32_t* pos_ptr, const uint32_t* cu,
