@@ -663,12 +663,12 @@ ROW_SHAPES = [  # (n_head, n_kv, head_dim, block_tokens)
 @pytest.mark.parametrize("dtype", [KvDataType.F32, KvDataType.F16, KvDataType.BF16])
 @pytest.mark.parametrize("shape", ROW_SHAPES, ids=lambda s: "x".join(map(str, s)))
 def test_row_kernels_edges(dev, dtype, shape):
-    """The row kernels (head_dim 64 / 128, power-of-two pages) at lengths around
-    their tiles, waves and splits, head groups of 1 to 17, NaN in every slot no
-    sequence owns and an invalid table entry, split lengths that are one tile,
-    several, and none of theirs (the per-token kernel).  K and V are exact in
-    either and the weights keep 22 bits or more, so f32's bound, 1e-5 max-abs,
-    holds for every type."""
+    """The row kernels (head_dim 64 / 128, power-of-two pages; the per-token kernel on
+    the shapes that keep it) at lengths around their tiles, waves and splits, head
+    groups of 1 to 17, NaN in every slot no sequence owns and an invalid table
+    entry, split lengths that are one tile, several, and none of theirs (the
+    per-token kernel).  K and V are exact in either and the weights keep 24 bits, so
+    f32's bound, 1e-5 max-abs, holds for every type."""
     n_head, n_kv, hd, bt = shape
     rng = np.random.default_rng(sum(shape))
     lens = np.array([0, 1, 31, 32, 33, 127, 128, 129, 257, 640], np.int64)
@@ -724,9 +724,10 @@ def test_row_kernels_edges(dev, dtype, shape):
 @pytest.mark.parametrize("dtype", [KvDataType.F32, KvDataType.F16, KvDataType.BF16])
 @pytest.mark.parametrize("shape", ROW_SHAPES, ids=lambda s: "x".join(map(str, s)))
 def test_row_kernels_fused_step(dev, dtype, shape):
-    """The fused single-sequence step of the row kernels on a page no one has
-    written (NaN): positions that open a page, a tile and a split, and one
-    behind a masked page entry, whose row must not be written."""
+    """The fused single-sequence step of the row kernels (small pages: of the per-token
+    kernel where it is kept) on a page no one has written (NaN): positions that open
+    a page, a tile and a split, and one behind a masked page entry, whose row must
+    not be written."""
     n_head, n_kv, hd, bt = shape
     rl = n_kv * hd
     rng = np.random.default_rng(hd + bt)

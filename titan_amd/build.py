@@ -4,7 +4,8 @@ Outputs (git-ignored, shipped in-tree to the GPU box):
   titan_amd/lib/paged_kv.hsaco      append / gather / page copy / table kernels
   titan_amd/lib/paged_decode_{f32,f16,bf16}.hsaco  split-K decode attention
   titan_amd/lib/paged_prefill.hsaco  MFMA causal chunked prefill
-  titan_amd/lib/paged_rows.hsaco     the same for a few query rows (key split)
+  titan_amd/lib/paged_rows.hsaco     key-split MFMA kernels: prefill of a few query
+      rows, fixed-split decode
   titan_amd/lib/paged_decode_tiles_{f16,bf16,fp8}.hsaco  token-balanced decode
       (MFMA q.k, optional fused append)
   titan_amd/lib/libengine_hip.so    hipModuleLoad / hipModuleLaunchKernel C-ABI

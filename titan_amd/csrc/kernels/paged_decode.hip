@@ -7,8 +7,10 @@
 // tokens t < n with scores q.k * 1/sqrt(head_dim); out = softmax-weighted V.
 //
 // This kernel serves the head sizes, page sizes and splits that the MFMA row
-// kernels (eh_decode_rows_*, paged_rows.hip) do not take, and f32 batches at
-// head_dim 128; eh_decode_merge combines the partials of both.
+// kernels (eh_decode_rows_*, paged_rows.hip) do not take, and the shapes it is
+// faster on: f32 batches at head_dim 128 and, with few q heads per kv head, most
+// pages under 8 tokens and large f32 batches at head_dim 64 (the launcher's
+// pick_decode_kernel); eh_decode_merge combines the partials of both.
 //
 // Work decomposition (MI355X-first, not the reference's warp-per-q-head):
 //   * one workgroup (4 waves) per (context split, kv head [x head chunk], sequence);
